@@ -50,6 +50,8 @@ template <> struct Mfma<double> {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
+  // the row of operand lane i that puts row 4 g + r in register r of lane group g
+  static __device__ __forceinline__ int solve_row(int i) { return 4 * (i & 3) + (i >> 2); }
 };
 template <> struct Mfma<float> {
   using acc = v4f;
@@ -58,6 +60,7 @@ template <> struct Mfma<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  static __device__ __forceinline__ int solve_row(int i) { return i; }
 };
 
 // C[i][j] += alpha * sum_k A[i][k] B[k][j] for one BM x BN tile at
@@ -855,9 +858,9 @@ __device__ __forceinline__ void tile_mac(TileAcc<T> &tot, int K, TileMem<T> &sm,
 // Each block row is one left-looking launch over the batch: a workgroup
 // accumulates F[block, done rows] Z[done rows, 64 columns] in registers,
 // subtracts it from the right-hand side and solves with the 128 x 128
-// diagonal block in 32-row slices (products with the inverted 32 x 32
-// triangles), so X is read and written once per phase.  4/3 n^3 flop; bound by the matrix cores where the batch
-// fills the chip.  (Rank-32 updates of all of X after each 32-row solve took
+// diagonal block by substitution (block_solve), so X is read and written once
+// per phase.  4/3 n^3 flop; bound by the matrix cores where the batch fills the
+// chip.  (Rank-32 updates of all of X after each 32-row solve took
 // 2 n^3 flop and read and wrote X 72 times at order 2304: for 64 FP32
 // matrices of order 256..2304, 21.3 ms.)
 // Row permutation of the pivots: element v of the identity ends at position
@@ -893,47 +896,43 @@ __global__ void __launch_bounds__(256) k_perm(BatchView bv, const int *__restric
 constexpr int IB = CM;     // block rows of the inverse
 constexpr int INV_GS = 8;  // column tiles of a block row that share an XCD
 
-// x <- T^-1 e_c for the unit lower (or the upper) triangle T of 32 rows held
-// by columns, st[c * SST + r]; one lane per column.  In FP32 the next
-// column's coefficients are loaded before the current one's products (the scheduling
-// barriers keep all 496 from being loaded first: they would not fit the
-// registers).
-constexpr int SST = 34;
-template <typename T, bool UPPER>
-__device__ __forceinline__ void tri_inverse_col(const T *st, T (&x)[32])
+// x / u with r = 1 / u taken once for a column: the quotient corrected by its
+// residual (FP64) or formed in FP64 (FP32); where that is not finite, the
+// division itself.
+__device__ __forceinline__ double near_rcp(double u)
 {
-  constexpr bool AHEAD = sizeof(T) == 4;  // (in FP64 the registers do not hold two columns)
-  T cur[32], nxt[32];
-  auto load = [&](T(&v)[32], int c) {
-#pragma unroll
-    for (int r = 0; r < 32; r++)
-      if (UPPER ? r <= c : r > c) v[r] = st[c * SST + r];
-  };
-  if (AHEAD) load(cur, UPPER ? 31 : 0);
-#pragma unroll
-  for (int q = 0; q < 32; q++) {
-    const int c = UPPER ? 31 - q : q;
-    if (!AHEAD) load(cur, c);
-    else if (q < 31) load(nxt, UPPER ? c - 1 : c + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (UPPER) x[c] /= cur[c];
-#pragma unroll
-    for (int r = 0; r < 32; r++)
-      if (UPPER ? r < c : r > c) x[r] -= cur[r] * x[c];
-    if (AHEAD) {
-#pragma unroll
-      for (int r = 0; r < 32; r++) cur[r] = nxt[r];
-    }
-  }
+  double r = __builtin_amdgcn_rcp(u);
+  r = __builtin_fma(r, __builtin_fma(-u, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-u, r, 1.0), r);
+}
+__device__ __forceinline__ double quot(double x, double u, double r)
+{
+  double q = x * r;
+  q = __builtin_fma(r, __builtin_fma(-u, q, x), q);
+  if (!(fabs(q) <= 1.7976931348623157e308)) q = x / u;
+  return q;
+}
+__device__ __forceinline__ float quot(float x, float u, double r)
+{
+  float q = (float)((double)x * r);
+  if (!(fabsf(q) <= 3.4028234663852886e38f)) q = x / u;
+  return q;
 }
 
 // out <- T^-1 acc for the 128 x 64 tile of right-hand sides in acc and the
-// triangle T (unit lower, or upper) of order jb <= 128 at D: 32-row slices in
-// turn, each a product with the slice's inverted 32 x 32 triangle (four
-// inverted at once, one per wave) followed by the update of the slices to
-// come.  `sol` is SOL<T> elements of LDS: the slice before (sX) and after (sY)
-// its solve, and the four triangles.
-template <typename T> constexpr int SOL = 4 * 32 * SST + 2 * 32 * (CN + 1);
+// triangle T (unit lower, or upper) of order jb <= 128 at D, by substitution:
+// 32-row slices in turn, each followed by the update of the slices to come.
+// In a slice, wave w solves 16 of the columns.  Lane (l15, g = l / 16) holds
+// rows 4 g .. 4 g + 3 of column l15 of each 16-row tile: group b's turn comes
+// with every earlier row subtracted, it substitutes in its 4 x 4 triangle, and
+// its four rows go out to the later groups one product each (the other groups'
+// rows enter as 0, so nothing but these rows is multiplied).  Products with
+// inverted triangles of 32 rows took the same time, with residuals larger by
+// 7-20 % on bag matrices and without bound where a triangle is ill-conditioned.
+// `sol` is SOL<T, MF> elements of LDS: the slice before (sX) and after (sY) its
+// solve, the four triangles, and (vector ALUs) the waves' blocks of T.
+constexpr int SST = 34;
+template <typename T, bool MF> constexpr int SOL = (MF ? 4 : 8) * 32 * SST + 2 * 32 * (CN + 1);
 template <typename T, bool MF, bool UPPER>
 __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld, int jb, T *sol,
                                             T *out, long ldo, int cols)
@@ -943,8 +942,7 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
   const int l15 = lane & 15, l4 = lane >> 4;
   T *const sT = sol, *const sX = sol + 4 * ST, *const sY = sX + SX;
   {
-    // the wave's diagonal block (identity past the matrix), by columns, and
-    // its inverse: four blocks at once, one per wave
+    // the wave's diagonal block, identity past the matrix
     T *const st = sT + wv * ST;
     const TileSrc<T> Dw{D + (long)(wv * 32) * ld + wv * 32, ld, jb - wv * 32, jb - wv * 32};
     T v[16];
@@ -953,20 +951,13 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
 #pragma unroll
     for (int q = 0; q < 16; q++) {
       const int r = 2 * q + (lane >> 5), c = lane & 31;
-      st[c * SST + r] = r == c && wv * 32 + r >= jb ? (T)1 : v[q];
+      st[r * SST + c] = r == c && wv * 32 + r >= jb ? (T)1 : v[q];
     }
-    __builtin_amdgcn_wave_barrier();
-    T x[32];
-#pragma unroll
-    for (int r = 0; r < 32; r++) x[r] = r == (lane & 31) ? (T)1 : (T)0;
-    tri_inverse_col<T, UPPER>(st, x);
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int r = 0; r < 32; r++) st[r * SST + (lane & 31)] = x[r];  // by rows
   }
 #pragma unroll 1
   for (int q = 0; q < 4; q++) {
     const int s = UPPER ? 3 - q : q;  // the slice solved now, held by wave s
+    if (s * 32 >= jb) continue;
     if (wv == s) {
 #pragma unroll
       for (int a = 0; a < 2; a++)
@@ -986,35 +977,101 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
 #pragma unroll
         for (int a = 0; a < 2; a++) av[kk][a] = E.get(0, a * 16 + l15, 0, kk * 4 + l4);
     __syncthreads();
-    // y = T_s^-1 x, 16 columns per wave
-    typename Mfma<T>::acc y[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
     const T *const ti = sT + s * ST;
     if constexpr (MF) {
+      const int col = wv * 16 + l15;
+      const int ar = Mfma<T>::solve_row(l15);  // the row that operand lane l15 stands for
+      typename Mfma<T>::acc x[2];
 #pragma unroll
-      for (int kk = 0; kk < 8; kk++) {
-        const T xv = sX[(kk * 4 + l4) * SXW + wv * 16 + l15];
+      for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int a = 0; a < 2; a++)
-          y[a] = Mfma<T>::op(ti[(a * 16 + l15) * SST + kk * 4 + l4], xv, y[a]);
+        for (int r = 0; r < 4; r++) x[a][r] = sX[(a * 16 + 4 * l4 + r) * SXW + col];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int a = UPPER ? 1 - h : h;
+        const T *const ta = ti + a * 16 * SST + a * 16;  // the tile's triangle
+        T d[4][4], v[4];
+        double rc[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            if (UPPER ? j >= i : j < i) d[i][j] = ta[(4 * l4 + i) * SST + 4 * l4 + j];
+          v[i] = ta[ar * SST + 4 * l4 + i];
+          v[i] = (UPPER ? (ar >> 2) < l4 : (ar >> 2) > l4) ? -v[i] : (T)0;
+          if (UPPER) rc[i] = near_rcp((double)d[i][i]);
+        }
+        if (h == 1) {  // the other tile's rows, in the wave's columns of sY
+          const int o = UPPER ? 16 : 0;
+#pragma unroll
+          for (int kk = 0; kk < 4; kk++)
+            x[a] = Mfma<T>::op(-ti[(a * 16 + ar) * SST + o + kk * 4 + l4],
+                               sY[(o + kk * 4 + l4) * SXW + col], x[a]);
+        }
+        T res[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const int b = UPPER ? 3 - g : g;
+          T y[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int r = UPPER ? 3 - i : i;
+            y[r] = x[a][r];
+#pragma unroll
+            for (int j = 0; j < i; j++) {
+              const int c = UPPER ? 3 - j : j;
+              y[r] -= d[r][c] * y[c];
+            }
+            if (UPPER) y[r] = quot(y[r], d[r][r], rc[r]);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) res[r] = l4 == b ? y[r] : res[r];
+          if (g < 3)
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[a] = Mfma<T>::op(v[r], l4 == b ? y[r] : (T)0, x[a]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int row = a * 16 + 4 * l4 + r;
+          sY[row * SXW + col] = res[r];
+          if (s * 32 + row < jb && col < cols) out[(long)(s * 32 + row) * ldo + col] = res[r];
+        }
+        __builtin_amdgcn_wave_barrier();
       }
     } else {
-      for (int k = 0; k < 32; k++) {
-        const T xv = sX[k * SXW + wv * 16 + l15];
+      // wave w holds rows 8 w .. 8 w + 7 of every column
+      T x[8];
 #pragma unroll
-        for (int a = 0; a < 2; a++)
+      for (int r = 0; r < 8; r++) x[r] = sX[(wv * 8 + r) * SXW + lane];
+#pragma unroll 1
+      for (int g = 0; g < 4; g++) {
+        const int b = UPPER ? 3 - g : g;
+        const T *const tb = ti + wv * 8 * SST + b * 8;  // the wave's rows, wave b's columns
+        if (wv == b) {
 #pragma unroll
-          for (int r = 0; r < 4; r++)
-            y[a][r] += ti[(a * 16 + Mfma<T>::row(lane, r)) * SST + k] * xv;
+          for (int i = 0; i < 8; i++) {
+            const int r = UPPER ? 7 - i : i;
+#pragma unroll
+            for (int j = 0; j < i; j++) {
+              const int c = UPPER ? 7 - j : j;
+              x[r] -= tb[r * SST + c] * x[c];
+            }
+            if (UPPER) x[r] /= tb[r * SST + r];
+            const int row = b * 8 + r;
+            sY[row * SXW + lane] = x[r];
+            if (s * 32 + row < jb && lane < cols) out[(long)(s * 32 + row) * ldo + lane] = x[r];
+          }
+        }
+        __syncthreads();
+        if (UPPER ? wv < b : wv > b)
+#pragma unroll
+          for (int c = 0; c < 8; c++) {
+            const T yc = sY[(b * 8 + (UPPER ? 7 - c : c)) * SXW + lane];
+#pragma unroll
+            for (int r = 0; r < 8; r++) x[r] -= tb[r * SST + (UPPER ? 7 - c : c)] * yc;
+          }
       }
     }
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = a * 16 + Mfma<T>::row(lane, r), col = wv * 16 + l15;
-        sY[row * SXW + col] = y[a][r];
-        if (s * 32 + row < jb && col < cols) out[(long)(s * 32 + row) * ldo + col] = y[a][r];
-      }
     __syncthreads();
     if (later) {  // acc -= F[own slice, solved slice] y
       TileAcc<T> part;
@@ -1034,12 +1091,19 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
             for (int c = 0; c < 4; c++) part[a][c] = Mfma<T>::op(av[kk][a], yv[c], part[a][c]);
         }
       } else {
+        T *const se = sY + SX + wv * ST;  // the wave's own
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++)
+#pragma unroll
+          for (int a = 0; a < 2; a++) se[(a * 16 + l15) * SST + kk * 4 + l4] = av[kk][a];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 2
         for (int k = 0; k < 32; k++)
 #pragma unroll
           for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-              const T v = E.get(0, a * 16 + Mfma<T>::row(lane, r), 0, k);
+              const T v = se[(a * 16 + Mfma<T>::row(lane, r)) * SST + k];
 #pragma unroll
               for (int c = 0; c < 4; c++) part[a][c][r] += v * sY[k * SXW + c * 16 + l15];
             }
@@ -1055,13 +1119,13 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
 // Block row t (from the top, or from the bottom when UPPER) of Z for every
 // matrix that has one.
 template <typename T, bool MF, bool UPPER>
-__global__ void __launch_bounds__(256, 2) k_inv_rows(const T *LU, T *X, BatchView bv, int t,
+__global__ void __launch_bounds__(256, MF ? 2 : 1) k_inv_rows(const T *LU, T *X, BatchView bv, int t,
                                                      int ng)
 {
   // the solve's LDS follows the product's in the same memory
   __shared__ __align__(16) union {
     TileMem<T> mem;
-    T sol[SOL<T>];
+    T sol[SOL<T, MF>];
   } sh;
   const XcdTile xt = xcd_tile<INV_GS>(blockIdx.x, ng);
   const int b = xt.b;
@@ -1111,10 +1175,10 @@ __global__ void __launch_bounds__(256, 2) k_inv_rows(const T *LU, T *X, BatchVie
 // the other, and U12 by four 32-row solves and updates in between, took 175 us
 // for the first block of 64 FP64 matrices of order 256..2304; this takes 131.)
 template <typename T, bool MF>
-__global__ void __launch_bounds__(256, 2) k_lu_right(T *base, BatchView bv, const int *pivb, int k)
+__global__ void __launch_bounds__(256, MF ? 2 : 1) k_lu_right(T *base, BatchView bv, const int *pivb, int k)
 {
   __shared__ int pv[LOB], dst[2 * LOB], src[2 * LOB];
-  __shared__ __align__(16) T sol[SOL<T>];
+  __shared__ __align__(16) T sol[SOL<T, MF>];
   static_assert(LOB == CM && LOB == 128, "a block is a tile's rows");
   const int b = blockIdx.y;
   const int n = bv.n[b];
