@@ -10,7 +10,7 @@
 //
 // LU: right-looking with partial pivoting (the factors equal those of
 // LAPACK's whole-row interchanges).  Up to order PR*PT, blocks of LOB = 128
-// columns, each factored as register panels of 16 or 32 columns, which also
+// columns, each factored as register panels of 16 (FP64) or 32 columns, which also
 // interchange the block's other columns and solve for U to their right
 // (k_lu_panel_reg), and updates inside the block (k_lu_update); then, outside
 // it, one launch for all interchanges of the block and U12 = L11^{-1} A12
@@ -242,6 +242,7 @@ __global__ void __launch_bounds__(256) k_lu_panel(T *base, BatchView bv, int *pi
 constexpr int PT = 1024;  // most threads of the register panel
 constexpr int PR = 3;     // panel rows per thread
 constexpr int LOB = 128;  // outer block of the register-panel LU
+template <typename T> constexpr int PW = sizeof(T) == 8 ? 16 : 32;  // panel columns
 
 // DPP move of a lane's unsigned value; lanes the move does not write get 0.
 template <int CTRL, int ROW_MASK>
@@ -375,7 +376,7 @@ __device__ __forceinline__ int swap_source(int dst, int k, int jb, const int *pv
   return pos;
 }
 
-// Panel of W columns held in registers: one block of NT threads per matrix
+// Panel of W = PW columns held in registers: one block of NT threads per matrix
 // (256, 512 or 1024, the fewest that hold the rows left), row k + t + q*NT of
 // the panel in thread t, slot q < PR (orders up to PR*PT).  Rows stay where
 // they are; an interchange exchanges their positions (pos, from k).  Per
@@ -393,14 +394,15 @@ __device__ __forceinline__ int swap_source(int dst, int k, int jb, const int *pv
 // per column, the pivot's row in scalar registers and no exchange of rows: for
 // 64 matrices of order 256..2304 an FP64 panel of 16 columns with 1024 threads
 // 55 -> 47 us, and with the block's interchanges and U, which were a launch of
-// 8-12 us; with 256 and 512 threads two panels of 16 (62 and 88 us) -> one of
-// 32 (55 and 72).
-template <typename T, int W, int NT>
+// 8-12 us.  (FP64 panels of 32 columns with up to 512 threads saved a tenth of
+// their time, but a row takes 32 one-column updates in turn instead of 16 and a
+// product: |A - L U| grew by 6 % on bag matrices.)
+template <typename T, int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT / 256)))
 k_lu_panel_reg(T *base, BatchView bv, int *pivb, int *info,
                                                      int k, int k0, int k1)
 {
-  constexpr int NW = NT / 64;
+  constexpr int NW = NT / 64, W = PW<T>;
   static_assert(NW <= 16 && NT >= 2 * LOB && 2 * W <= NT, "posts in a row of lanes; the gather");
   // double-buffered by column parity: a buffer is rewritten two columns
   // later, after every thread has passed the barrier between
@@ -1466,11 +1468,11 @@ void launch_update(th2d_ctx *c, bool mf, T *A, BatchView bv, int count, int kk, 
     hipLaunchKernelGGL((k_lu_update<T, false>), g, dim3(256), 0, st, A, bv, kk, K, r0, r1, c0, c1);
 }
 
-template <typename T, int W, int NT>
+template <typename T, int NT>
 void launch_panel(th2d_ctx *c, T *A, BatchView bv, int count, int *piv, int *info, int kk, int k,
                   int ce)
 {
-  hipLaunchKernelGGL((k_lu_panel_reg<T, W, NT>), dim3(count), dim3(NT), 0, c->stream, A, bv, piv,
+  hipLaunchKernelGGL((k_lu_panel_reg<T, NT>), dim3(count), dim3(NT), 0, c->stream, A, bv, piv,
                      info, kk, k, ce);
 }
 
@@ -1480,15 +1482,13 @@ void lu_blocks(th2d_ctx *c, const th2d_batch *bt, T *A, int *piv, int *info)
   const BatchView bv = view(bt);
   const int N = bt->max_n, cnt = bt->count;
   constexpr int END = 1 << 30;  // a range bound past every order
-  constexpr int WL = sizeof(T) == 8 ? 16 : 32;
+  constexpr int W = PW<T>;
   for (int k = 0; k < N; k += LOB) {
     const int ce = std::min(k + LOB, N), rows = N - k;  // the most rows a matrix has left
-    // (32 FP64 columns need 192 registers: up to 512 threads)
-    const int W = rows <= PR * 512 ? 32 : WL;
     for (int kk = k; kk < ce; kk += W) {
-      if (rows <= PR * 256) launch_panel<T, 32, 256>(c, A, bv, cnt, piv, info, kk, k, ce);
-      else if (rows <= PR * 512) launch_panel<T, 32, 512>(c, A, bv, cnt, piv, info, kk, k, ce);
-      else launch_panel<T, WL, PT>(c, A, bv, cnt, piv, info, kk, k, ce);
+      if (rows <= PR * 256) launch_panel<T, 256>(c, A, bv, cnt, piv, info, kk, k, ce);
+      else if (rows <= PR * 512) launch_panel<T, 512>(c, A, bv, cnt, piv, info, kk, k, ce);
+      else launch_panel<T, PT>(c, A, bv, cnt, piv, info, kk, k, ce);
       const int cb = kk + W;
       if (cb < ce) launch_update<T>(c, MF, A, bv, cnt, kk, W, cb, END, cb, ce, N);
     }
