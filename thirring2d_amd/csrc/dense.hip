@@ -396,11 +396,12 @@ __device__ __forceinline__ int swap_source(int dst, int k, int jb, const int *pv
 // 55 -> 47 us, and with the block's interchanges and U, which were a launch of
 // 8-12 us.  (FP64 panels of 32 columns with up to 512 threads saved a tenth of
 // their time, but a row takes 32 one-column updates in turn instead of 16 and a
-// product: |A - L U| grew by 6 % on bag matrices.)
+// product: |A - L U| grew by 6 % on bag matrices.)  116..128 registers and 38 KB
+// of LDS with 256 threads let four matrices share a CU: 1000 FP64 matrices of
+// order 64 take 179 us (402 with one per CU).
 template <typename T, int NT>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT / 256)))
-k_lu_panel_reg(T *base, BatchView bv, int *pivb, int *info,
-                                                     int k, int k0, int k1)
+__global__ void __launch_bounds__(NT)
+k_lu_panel_reg(T *base, BatchView bv, int *pivb, int *info, int k, int k0, int k1)
 {
   constexpr int NW = NT / 64, W = PW<T>;
   static_assert(NW <= 16 && NT >= 2 * LOB && 2 * W <= NT, "posts in a row of lanes; the gather");
