@@ -713,25 +713,43 @@ __global__ void __launch_bounds__(256) k_lu_logdet(const T *base, BatchView bv, 
 constexpr int CM = 128, CN = 64, CK = 16, CNP = CN + 16;
 
 // Workgroups go to the 8 XCDs in turn, and each XCD has its own L2: groups
-// of GS tiles that read the same rows of a factor are given to one XCD
+// of gs tiles that read the same rows of a factor are given to one XCD
 // (consecutive workgroups of it), so that the rows are fetched once per group
 // instead of once per tile.  Workgroup id -> tile `w` of group `g` of matrix
 // b, for `ng` groups per matrix; xcd_grid gives the number of workgroups.
 struct XcdTile {
   int b, g, w;
 };
-template <int GS> __device__ __forceinline__ XcdTile xcd_tile(unsigned id, int ng)
+__device__ __forceinline__ XcdTile xcd_tile(unsigned id, int gs, int ng)
 {
   const unsigned r = id >> 3;
-  const int gid = (int)(r / GS) * 8 + (int)(id & 7), b = gid / ng;
+  const int gid = (int)(r / (unsigned)gs) * 8 + (int)(id & 7), b = gid / ng;
   // (rotated by the matrix: else, with ng even, a partly empty last group of
   // every matrix would fall on the same XCDs)
-  return XcdTile{b, (gid + b) % ng, (int)(r % GS)};
+  return XcdTile{b, (gid + b) % ng, (int)(r % (unsigned)gs)};
 }
-inline unsigned xcd_grid(int GS, int ng, int count)
+inline unsigned xcd_grid(int gs, int ng, int count)
 {
-  return (unsigned)((((long)ng * count + 7) / 8) * 8 * GS);
+  return (unsigned)((((long)ng * count + 7) / 8) * 8 * gs);
 }
+
+// tx x ty tiles in gx x gy groups of sx x sy, at most 8 x 8 tiles to a group
+// (and no more than there are: a group's unused tiles are workgroups too).
+struct TileGroups {
+  int gx, gy, sx, sy;
+  TileGroups(int tx, int ty)
+      : gx((tx + 7) / 8), gy((ty + 7) / 8), sx(std::min(tx, 8)), sy(std::min(ty, 8))
+  {
+  }
+  unsigned grid(int count) const { return xcd_grid(sx * sy, gx * gy, count); }
+  __device__ __forceinline__ XcdTile tile(unsigned id, int &row, int &col) const
+  {
+    const XcdTile xt = xcd_tile(id, sx * sy, gx * gy);
+    row = xt.g / gx * sy + xt.w / sx;
+    col = xt.g % gx * sx + xt.w % sx;
+    return xt;
+  }
+};
 
 template <typename T> struct TileMem {
   T a[2][CM * (CK + 1)];
@@ -897,7 +915,6 @@ __global__ void __launch_bounds__(256) k_perm(BatchView bv, const int *__restric
 }
 
 constexpr int IB = CM;     // block rows of the inverse
-constexpr int INV_GS = 8;  // column tiles of a block row that share an XCD
 
 // x / u with r = 1 / u taken once for a column: the quotient corrected by its
 // residual (FP64) or formed in FP64 (FP32); where that is not finite, the
@@ -1123,20 +1140,20 @@ __device__ __forceinline__ void block_solve(TileAcc<T> &acc, const T *D, long ld
 // matrix that has one.
 template <typename T, bool MF, bool UPPER>
 __global__ void __launch_bounds__(256, MF ? 2 : 1) k_inv_rows(const T *LU, T *X, BatchView bv, int t,
-                                                     int ng)
+                                                     TileGroups tg)
 {
   // the solve's LDS follows the product's in the same memory
   __shared__ __align__(16) union {
     TileMem<T> mem;
     T sol[SOL<T, MF>];
   } sh;
-  const XcdTile xt = xcd_tile<INV_GS>(blockIdx.x, ng);
-  const int b = xt.b;
+  int tr, tc;
+  const int b = tg.tile(blockIdx.x, tr, tc).b;
   if (b >= bv.count) return;
   const int n = bv.n[b];
   const int nb = (n + IB - 1) / IB;
   if (t >= nb) return;
-  const int k0 = (UPPER ? nb - 1 - t : t) * IB, j0 = (xt.g * INV_GS + xt.w) * CN;
+  const int k0 = (UPPER ? nb - 1 - t : t) * IB, j0 = tc * CN;
   if (j0 >= n || (!UPPER && j0 >= k0 + IB)) return;  // (L^-1 is 0 there)
   const int jb = min(IB, n - k0);
   const T *F = LU + bv.off[b];
@@ -1169,6 +1186,98 @@ __global__ void __launch_bounds__(256, MF ? 2 : 1) k_inv_rows(const T *LU, T *X,
   __syncthreads();  // the product's LDS is free
   block_solve<T, MF, UPPER>(acc, F + (long)k0 * n + k0, n, jb, sh.sol, Z + (long)k0 * n + j0, n,
                             n - j0);
+}
+
+// The inverse of matrices of order n <= 64, one wave each: lane l solves for
+// column l of Z = U^-1 L^-1, four rows at a time from the rows before (LU and Z
+// in LDS, the coefficients the same in every lane), and with `permute` writes
+// it as the column of A^-1 it is.  Bound by LDS reads and their latency.  A
+// workgroup of k_inv_rows per matrix and phase is mostly idle at such orders:
+// 1000 FP64 matrices of order 16 take 30 us here (431 in k_inv_rows with groups
+// of eight tiles), of order 64 172 (468).  A few matrices of order above 32 are
+// better off there: one of order 64 takes 49 us, 77 here.
+constexpr int IS = 64;
+inline bool small_inverse(const th2d_ctx *c, const th2d_batch *bt)
+{
+  return bt->max_n <= 32 || (bt->max_n <= IS && bt->count > c->num_cu);
+}
+template <typename T>
+__global__ void __launch_bounds__(64) k_inv_small(const T *LU, T *X, BatchView bv, const int *pivb,
+                                                  int nmax, int permute)
+{
+  extern __shared__ double is_raw[];
+  const int b = blockIdx.x, lane = threadIdx.x;
+  const int n = bv.n[b];
+  if (n < 1 || n > nmax) return;  // (nmax <= IS)
+  const int m = (n + 3) & ~3;  // identity beyond n
+  T *S = (T *)is_raw, *Z = S + m * m;
+  const T *F = LU + bv.off[b];
+  for (int e = lane; e < m * m; e += 64) {
+    const int r = e / m, c = e - r * m;
+    S[e] = r < n && c < n ? F[r * n + c] : (r == c ? (T)1 : (T)0);
+  }
+  __syncthreads();
+  if (lane < m) {
+    T *z = Z + lane;
+    for (int i = 0; i < m; i += 4) {  // L z = e_lane
+      const T *si = S + i * m;
+      T x[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) x[t] = i + t == lane ? (T)1 : (T)0;
+      for (int q = 0; q < i; q += 4)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const T y = z[(q + u) * m];
+#pragma unroll
+          for (int t = 0; t < 4; t++) x[t] -= si[t * m + q + u] * y;
+        }
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+#pragma unroll
+        for (int u = 0; u < t; u++) x[t] -= si[t * m + i + u] * x[u];
+        z[(i + t) * m] = x[t];
+      }
+    }
+    for (int i = m - 4; i >= 0; i -= 4) {  // U z = z
+      const T *si = S + i * m;
+      T x[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) x[t] = z[(i + t) * m];
+      for (int q = i + 4; q < m; q += 4)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const T y = z[(q + u) * m];
+#pragma unroll
+          for (int t = 0; t < 4; t++) x[t] -= si[t * m + q + u] * y;
+        }
+#pragma unroll
+      for (int t = 3; t >= 0; t--) {
+#pragma unroll
+        for (int u = 3; u > t; u--) x[t] -= si[t * m + i + u] * x[u];
+        x[t] /= si[t * m + i + t];
+        z[(i + t) * m] = x[t];
+      }
+    }
+  }
+  int col = lane;
+  if (permute) {
+    // element `lane` of the identity ends at position pos
+    const int *piv = pivb + bv.poff[b];
+    int pos = lane;
+    for (int j = 0; j < n; j++) {
+      const int p = piv[j];
+      pos = pos == j ? p : (pos == p ? j : pos);
+    }
+    __syncthreads();  // the factors have been read: their LDS holds the columns
+    int *pm = (int *)is_raw;
+    if (lane < n) pm[pos] = lane;
+    __syncthreads();
+    if (lane < n) col = pm[lane];
+  }
+  if (lane < n) {
+    T *Xb = X + bv.off[b] + col;
+    for (int r = 0; r < n; r++) Xb[r * n] = Z[r * m + lane];
+  }
 }
 
 // After the block of columns k .. k + 127: its interchanges on 64 of the
@@ -1246,15 +1355,15 @@ __global__ void __launch_bounds__(256, MF ? 2 : 1) k_lu_right(T *base, BatchView
 // A22 -= L21 U12 beyond the block of columns k .. k + 127, one 128 x 64 tile
 // per workgroup; 8 x 8 tiles of a matrix share an XCD, and with it the rows of
 // L21 and the columns of U12.
-constexpr int TG = 8;
 template <typename T, bool MF>
-__global__ void __launch_bounds__(256, 2) k_lu_trail(T *base, BatchView bv, int k, int gx, int gy)
+__global__ void __launch_bounds__(256, 2) k_lu_trail(T *base, BatchView bv, int k, TileGroups tg)
 {
   __shared__ TileMem<T> mem;
-  const XcdTile xt = xcd_tile<TG * TG>(blockIdx.x, gx * gy);
+  int tr, tc;
+  const XcdTile xt = tg.tile(blockIdx.x, tr, tc);
   if (xt.b >= bv.count) return;
   const int n = bv.n[xt.b], ce = k + LOB;
-  const int i0 = ce + (xt.g / gx * TG + xt.w / TG) * CM, j0 = ce + (xt.g % gx * TG + xt.w % TG) * CN;
+  const int i0 = ce + tr * CM, j0 = ce + tc * CN;
   if (i0 >= n || j0 >= n) return;
   T *A = base + bv.off[xt.b];
   const int lane = threadIdx.x & 63, wr = (threadIdx.x >> 6) * 32, l15 = lane & 15;
@@ -1353,25 +1462,26 @@ __global__ void k_f64_to_f32_n(float *d, const double *s, long n)
 // registers, so L U never goes to memory.  (Promoting L and U to dense FP64
 // matrices first and reading the product back for the trace took 5.4 ms for
 // 64 matrices of order 256..2304, 2.8 of them the product.)
-constexpr int RT = 8;  // tiles of an 8 x 8 group share an XCD: L rows and U columns
+// Tiles of a group share an XCD: L rows and U columns.
 template <bool MF>
 __global__ void __launch_bounds__(256, 2) k_refine_trace(const double *A, const float *LU32,
                                                          const float *Z, const int *permb,
                                                          BatchView bv, double *part, int nparts,
-                                                         int gx, int gy)
+                                                         TileGroups tg)
 {
   __shared__ union {
     TileMem<double> mem;
     float z[CN * (CM + 1)];
   } sh;
   __shared__ double red[4];
-  const XcdTile xt = xcd_tile<RT * RT>(blockIdx.x, gx * gy);
+  int tr, tc;
+  const XcdTile xt = tg.tile(blockIdx.x, tr, tc);
   const int b = xt.b;
   if (b >= bv.count) return;
   const int n = bv.n[b];
   const int tx = (n + CN - 1) / CN, ty = (n + CM - 1) / CM;
   // the deepest tiles first
-  const int ti = ty - 1 - (xt.g / gx * RT + xt.w / RT), tj = tx - 1 - (xt.g % gx * RT + xt.w % RT);
+  const int ti = ty - 1 - tr, tj = tx - 1 - tc;
   if (ti < 0 || tj < 0) return;
   const int tile = ti * tx + tj, i0 = ti * CM, j0 = tj * CN;
   const long off = bv.off[b];
@@ -1503,9 +1613,9 @@ void lu_blocks(th2d_ctx *c, const th2d_batch *bt, T *A, int *piv, int *info)
     if constexpr (sizeof(T) == 8) {
       launch_update<T>(c, MF, A, bv, cnt, k, LOB, ce, END, ce, END, N);
     } else {
-      const int gx = ((N - ce + CN - 1) / CN + TG - 1) / TG, gy = ((N - ce + CM - 1) / CM + TG - 1) / TG;
-      hipLaunchKernelGGL((k_lu_trail<T, MF>), dim3(xcd_grid(TG * TG, gx * gy, cnt)), dim3(256), 0,
-                         c->stream, A, bv, k, gx, gy);
+      const TileGroups tg((N - ce + CN - 1) / CN, (N - ce + CM - 1) / CM);
+      hipLaunchKernelGGL((k_lu_trail<T, MF>), dim3(tg.grid(cnt)), dim3(256), 0, c->stream, A, bv, k,
+                         tg);
     }
   }
 }
@@ -1545,19 +1655,32 @@ void inverse_rows(th2d_ctx *c, const th2d_batch *bt, const T *LU, T *X)
   const int N = bt->max_n, nb = (N + IB - 1) / IB;
   const int ct = (N + CN - 1) / CN;
   for (int t = 0; t < nb; t++) {
-    const int ng = (std::min(ct, (t + 1) * (IB / CN)) + INV_GS - 1) / INV_GS;
-    hipLaunchKernelGGL((k_inv_rows<T, MF, false>), dim3(xcd_grid(INV_GS, ng, bt->count)), dim3(256),
-                       0, c->stream, LU, X, bv, t, ng);
+    const TileGroups tg(std::min(ct, (t + 1) * (IB / CN)), 1);
+    hipLaunchKernelGGL((k_inv_rows<T, MF, false>), dim3(tg.grid(bt->count)), dim3(256), 0, c->stream,
+                       LU, X, bv, t, tg);
   }
-  const int ng = (ct + INV_GS - 1) / INV_GS;
+  const TileGroups tg(ct, 1);
   for (int t = 0; t < nb; t++)
-    hipLaunchKernelGGL((k_inv_rows<T, MF, true>), dim3(xcd_grid(INV_GS, ng, bt->count)), dim3(256),
-                       0, c->stream, LU, X, bv, t, ng);
+    hipLaunchKernelGGL((k_inv_rows<T, MF, true>), dim3(tg.grid(bt->count)), dim3(256), 0, c->stream,
+                       LU, X, bv, t, tg);
+}
+
+template <typename T>
+void inverse_small(th2d_ctx *c, const th2d_batch *bt, const T *LU, const int *piv, T *X,
+                   int permute)
+{
+  const int m = (bt->max_n + 3) & ~3;
+  hipLaunchKernelGGL(k_inv_small<T>, dim3(bt->count), dim3(64), 2 * sizeof(T) * m * m, c->stream, LU,
+                     X, view(bt), piv, bt->max_n, permute);
 }
 
 template <typename T>
 void inverse_unpermuted(th2d_ctx *c, const th2d_batch *bt, const T *LU, T *X)
 {
+  if (small_inverse(c, bt)) {
+    inverse_small<T>(c, bt, LU, nullptr, X, 0);
+    return;
+  }
   if (use_mfma()) inverse_rows<T, true>(c, bt, LU, X);
   else inverse_rows<T, false>(c, bt, LU, X);
 }
@@ -1578,6 +1701,11 @@ int inverse_launch(th2d_ctx *c, const th2d_batch *bt, const T *LU, const int *pi
   const BatchView bv = view(bt);
   const int N = bt->max_n;
   if (N < 1) return TH2D_OK;
+  if (small_inverse(c, bt)) {
+    inverse_small<T>(c, bt, LU, piv, X, 1);
+    TH2D_HIP(hipGetLastError());
+    return TH2D_OK;
+  }
   inverse_unpermuted<T>(c, bt, LU, X);
   if (sizeof(T) * (size_t)N <= PERM_LDS) {
     perm_launch(c, bt, piv, perm, pstride);
@@ -1702,14 +1830,14 @@ extern "C" int th2d_lu_logdet_refined(th2d_ctx *c, const th2d_batch *b, const do
   const BatchView bv = view(b);
   inverse_unpermuted<float>(c, b, LU32, Z);
   perm_launch(c, b, piv, perm, 0);
-  const int gx = ((nmax + CN - 1) / CN + RT - 1) / RT, gy = ((nmax + CM - 1) / CM + RT - 1) / RT;
-  const dim3 grid(xcd_grid(RT * RT, gx * gy, count));
+  const TileGroups tg((nmax + CN - 1) / CN, (nmax + CM - 1) / CM);
+  const dim3 grid(tg.grid(count));
   if (use_mfma())
     hipLaunchKernelGGL(k_refine_trace<true>, grid, dim3(256), 0, c->stream, A, LU32,
-                       (const float *)Z, (const int *)perm, bv, part, nparts, gx, gy);
+                       (const float *)Z, (const int *)perm, bv, part, nparts, tg);
   else
     hipLaunchKernelGGL(k_refine_trace<false>, grid, dim3(256), 0, c->stream, A, LU32,
-                       (const float *)Z, (const int *)perm, bv, part, nparts, gx, gy);
+                       (const float *)Z, (const int *)perm, bv, part, nparts, tg);
   hipLaunchKernelGGL(k_add_correction, dim3(count), dim3(256), 0, c->stream, part, nparts, bv,
                      info, logabs);
   TH2D_HIP(hipGetLastError());
