@@ -694,8 +694,8 @@ def main():
     dt_mx, res_mx, kms, kn, kbytes = run_hmc(H, N, size, N.PREC_MIXED, args.steps, args.warmup,
                                              nsteps=nsteps, lats=lats)
     on = C.c_int(0)
-    N.check(N.lib().th2d_cg_last_resident(H.Context.get().ptr, C.byref(on)), "cg_last_resident")
-    resident = bool(on.value)
+    N.check(N.lib().th2d_cg_last_kernel(H.Context.get().ptr, C.byref(on)), "cg_last_kernel")
+    resident = on.value == 1
     tps = nch * args.steps / dt_mx
     acc = float(np.mean([r[1] for r in res_mx]))
     dH = np.array([r[0] for r in res_mx])

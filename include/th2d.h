@@ -185,9 +185,12 @@ int th2d_cg_last_tile(th2d_ctx *ctx, int *tt, int *tx);
  * step kernel when a cost model prices it faster, or when a tile is set
  * with th2d_set_cg_tile; FP64 batches of lattices of at most 2048 sites go
  * to the small-lattice kernel (th2d_set_cg_small).
- * th2d_cg_last_resident tells about the last inner solve: 1 every lattice
- * ran on whole regions of the resident kernel, 2 some did, 0 none did (the
- * step kernel, or uneven regions alone), 3 the small-lattice kernel. */
+ * th2d_cg_last_kernel tells which kernel ran the last inner solve: 0 the step
+ * kernel, 1 the resident kernel, 2 both (a split batch), 3 the small-lattice
+ * kernel.  th2d_cg_last_resident tells how many of its lattices it solved in
+ * the resident kernel and divide into whole regions (of 64 x 64 sites in FP32,
+ * 32 x 64 in FP64, or lie in one): 1 all, 2 some, 0 none; 3 the small-lattice
+ * kernel. */
 int th2d_set_cg_resident(th2d_ctx *ctx, int on);
 /* Step-kernel launches as captured graphs (0 off, default; 1 on): the
  * step kernel's iterations are issued as replays of a hipGraph holding 8
@@ -210,11 +213,12 @@ int th2d_set_cg_graph(th2d_ctx *ctx, int on);
  * ill-conditioned ones (m = 0.05: +13%), where the FP32 residual has drifted
  * by the end of a pass; hence off by default. */
 int th2d_set_cg_reliable(th2d_ctx *ctx, int on);
+int th2d_cg_last_kernel(th2d_ctx *ctx, int *kernel);
 int th2d_cg_last_resident(th2d_ctx *ctx, int *on);
 /* Small lattices (1, default; 0 off): an FP64 inner solve of a batch whose
  * lattices have at most 2048 sites runs as one launch, one workgroup per
  * lattice, the whole CG loop inside it (vectors in registers, the operator
- * through LDS); th2d_cg_last_resident then reports 3.  Off, or with a tile
+ * through LDS); th2d_cg_last_kernel then reports 3.  Off, or with a tile
  * set by th2d_set_cg_tile, the step kernel solves them.  Replaces no
  * reference function. */
 int th2d_set_cg_small(th2d_ctx *ctx, int on);

@@ -70,7 +70,8 @@ struct th2d_ctx {
   int cg_resident = 1;            // FP32 inner solves in the resident kernel when they fit
   int cg_reliable = 0;            // mixed solves continue the Krylov sequence across passes
   int res_capacity = -1;          // resident workgroups the device holds (-1: not queried)
-  int cg_last_resident = 0;       // the last inner solve: 0 step kernel, 1 resident, 2 both
+  int cg_last_kernel = 0;         // the last inner solve: 0 step kernel, 1 resident, 2 both, 3 small
+  int cg_last_resident = 0;       // and how many of its lattices divide into whole resident regions
   int hmc_graph = 1;              // small-lattice FP64 MD steps in one launch (0: one each)
   int cg_small = 1;               // FP64 solves of lattices up to 2048 sites in one launch
   long res_spin_limit = -1;       // polls of one resident-kernel wait (-1: the default)
