@@ -181,8 +181,9 @@ int th2d_cg_last_tile(th2d_ctx *ctx, int *tt, int *tx);
  * A lattice whose sides are not multiples of the regions' is cut into
  * regions of nearly equal sides; one larger than an XCD holds (32 regions)
  * is solved by the step kernel, and a batch that mixes such lattices with
- * others is split between the two kernels.  The whole batch goes to the
- * step kernel when a cost model prices it faster, or when a tile is set
+ * others is split between the two kernels where a cost model prices that
+ * faster.  The whole batch goes to the step kernel when it prices that
+ * faster, or when a tile is set
  * with th2d_set_cg_tile; FP64 batches of lattices of at most 2048 sites go
  * to the small-lattice kernel (th2d_set_cg_small).
  * th2d_cg_last_kernel tells which kernel ran the last inner solve: 0 the step

@@ -169,3 +169,20 @@ def test_fused_md_steps_match_the_general_ones(hmc, N, dims, mu, anti):
         assert np.max(np.abs(a1 - a0)) <= 2e-9
         assert np.max(np.abs(np.array(r1.acts) - np.array(r0.acts))) <= 2e-9 * np.sqrt(nt * nx)
         assert abs(r1.cg_iterations - r0.cg_iterations) <= max(4, r0.cg_iterations // 50)
+
+
+@pytest.mark.parametrize("dims, kernel", [
+    ([(512, 512), (64, 64), (96, 96)], BOTH),
+    ([(64, 64)] + [(384, 384)] + [(128, 128)] * 7, BOTH),
+    ([(384, 384), (96, 96)], STEP),          # the split would cost more than it saves
+    ([(16, 16), (384, 384)], STEP),
+])
+@pytest.mark.parametrize("prec", [0, 2])
+def test_split_batches(hmc, oracle, N, dims, kernel, prec):
+    """Lattices larger than an XCD's resident workgroups beside smaller ones."""
+    batch, rest = _batch(hmc, oracle, dims)
+    tol = 1e-12 if prec == 0 else 1e-10
+    xs, infos = batch.fmdm_invert_cg([b for _, _, b in rest],
+                                     hmc.cg_params(tol_rel=tol, precision=prec))
+    assert _kernel(N, batch.ctx) == kernel
+    _check(oracle, rest, xs, infos, tol)
