@@ -583,9 +583,9 @@ extern "C" int th2d_bag_batch_sweep(th2d_bag_batch *s, int nsteps, unsigned long
                 (unsigned)s->count);
   // runs of steps that the factors have room for (a step adds at most two),
   // each followed by the addition to B: between calls B is whole
-  for (int k = 0; k < nsteps; k += s->kmax / 2) {
+  for (long k = 0; k < nsteps; k += s->kmax / 2) {
     hipLaunchKernelGGL(k_bmc_steps, dim3((unsigned)s->count), dim3(BMC_NT), 0, c->stream, v, seed,
-                       counter + (unsigned long long)k, std::min(s->kmax / 2, nsteps - k),
+                       counter + (unsigned long long)k, (int)std::min<long>(s->kmax / 2, nsteps - k),
                        trace ? trace + (size_t)k * s->count : nullptr);
     hipLaunchKernelGGL(k_bmc_flush, gf, dim3(256), 0, c->stream, v);
   }

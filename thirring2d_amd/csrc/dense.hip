@@ -609,20 +609,20 @@ k_lu_panel_reg(T *base, BatchView bv, int *pivb, int *info, int k, int k0, int k
   }
 }
 
-// U12 = L11^{-1} A12 on rows k..k+jb-1 of the columns c0 <= c < c1 (all
-// from k + jb when c1 <= 0), unit lower L11 of order jb <= JB.  One thread
-// per column; its column of U12 lives in registers (the loops over the JB
+// U12 = L11^{-1} A12 on rows k..k+jb-1 of the columns from k + jb on, unit
+// lower L11 of order jb <= JB (the LDS panels' block rows).  One thread per
+// column; its column of U12 lives in registers (the loops over the JB
 // rows unroll fully, so every index is a constant), L11 in LDS.
 template <typename T, int JB>
-__global__ void __launch_bounds__(256) k_lu_trsm(T *base, BatchView bv, int k, int c0, int c1)
+__global__ void __launch_bounds__(256) k_lu_trsm(T *base, BatchView bv, int k)
 {
   __shared__ T sL[JB * JB];
   const int b = blockIdx.y;
   const int n = bv.n[b];
   if (k >= n) return;
   const int jb = min(JB, n - k);
-  const int cb = c1 > 0 ? c0 : k + jb, ce = c1 > 0 ? min(c1, n) : n;
-  if (cb >= ce) return;
+  const int cb = k + jb;
+  if (cb >= n) return;
   T *A = base + bv.off[b];
   for (int e = threadIdx.x; e < jb * jb; e += 256) {
     const int r = e / jb, q = e - r * jb;
@@ -630,7 +630,7 @@ __global__ void __launch_bounds__(256) k_lu_trsm(T *base, BatchView bv, int k, i
   }
   __syncthreads();
   const int c = cb + blockIdx.x * 256 + threadIdx.x;
-  if (c >= ce) return;
+  if (c >= n) return;
   T x[JB];
 #pragma unroll
   for (int r = 0; r < JB; r++) x[r] = r < jb ? A[(long)(k + r) * n + c] : (T)0;
@@ -1567,16 +1567,17 @@ BatchView view(const th2d_batch *b) { return BatchView{b->off, b->n, b->poff, b-
 
 template <typename T>
 void launch_update(th2d_ctx *c, bool mf, T *A, BatchView bv, int count, int kk, int K, int r0,
-                   int r1, int c0, int c1, int N, hipStream_t st = nullptr)
+                   int r1, int c0, int c1, int N)
 {
   const int rows = std::min(r1, N) - r0, cols = std::min(c1, N) - c0;
   if (rows <= 0 || cols <= 0) return;
-  if (!st) st = c->stream;
   dim3 g((cols + BN - 1) / BN, (rows + BM - 1) / BM, count);
   if (mf)
-    hipLaunchKernelGGL((k_lu_update<T, true>), g, dim3(256), 0, st, A, bv, kk, K, r0, r1, c0, c1);
+    hipLaunchKernelGGL((k_lu_update<T, true>), g, dim3(256), 0, c->stream, A, bv, kk, K, r0, r1, c0,
+                       c1);
   else
-    hipLaunchKernelGGL((k_lu_update<T, false>), g, dim3(256), 0, st, A, bv, kk, K, r0, r1, c0, c1);
+    hipLaunchKernelGGL((k_lu_update<T, false>), g, dim3(256), 0, c->stream, A, bv, kk, K, r0, r1, c0,
+                       c1);
 }
 
 template <typename T, int NT>
@@ -1638,7 +1639,7 @@ int lu_run(th2d_ctx *c, const th2d_batch *bt, T *A, int *piv, int *info)
       const int rest = N - k - NB;
       if (rest > 0) {
         hipLaunchKernelGGL((k_lu_trsm<T, NB>), dim3((rest + 255) / 256, cnt), dim3(256), 0,
-                           c->stream, A, bv, k, 0, 0);
+                           c->stream, A, bv, k);
         launch_update<T>(c, mf, A, bv, cnt, k, NB, k + NB, END, k + NB, END, N);
       }
     }
