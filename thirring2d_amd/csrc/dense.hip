@@ -946,9 +946,12 @@ __device__ __forceinline__ float quot(float x, float u, double r)
 // rows 4 g .. 4 g + 3 of column l15 of each 16-row tile: group b's turn comes
 // with every earlier row subtracted, it substitutes in its 4 x 4 triangle, and
 // its four rows go out to the later groups one product each (the other groups'
-// rows enter as 0, so nothing but these rows is multiplied).  Products with
-// inverted triangles of 32 rows took the same time, with residuals larger by
-// 7-20 % on bag matrices and without bound where a triangle is ill-conditioned.
+// rows enter as 0, so nothing but these rows is multiplied).  Bound by the
+// chain of these products, 24 per slice.  Products with inverted triangles of 32
+// rows took as long for the lower triangles and 7 % less per launch for the
+// upper ones (64 FP32 matrices of order 256..2304: 203 us, 218 here), with
+// residuals larger by 7-20 % on bag matrices and without bound where a triangle
+// is ill-conditioned.
 // `sol` is SOL<T, MF> elements of LDS: the slice before (sX) and after (sY) its
 // solve, the four triangles, and (vector ALUs) the waves' blocks of T.
 constexpr int SST = 34;
