@@ -59,6 +59,7 @@ def _check(oracle, rest, xs, infos, tol):
 @pytest.mark.parametrize("dims", [
     [(96, 96)], [(96, 96), (96, 160)], [(70, 66), (2, 66), (206, 116)],  # uneven alone
     [(96, 96), (128, 128), (32, 32)], [(96, 64)], [(128, 128)],
+    [(96, 96), (100, 70), (48, 130), (66, 66)] * 16,         # every XCD full, FP64 in two launches
 ])
 @pytest.mark.parametrize("prec", [0, 2])
 def test_resident_is_named(hmc, oracle, N, dims, prec):
